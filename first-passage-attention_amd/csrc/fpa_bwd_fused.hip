@@ -75,11 +75,14 @@ fpa_bwd_kvq_split_kernel(BwdParams p, BwdOrder ord, int nslots) {
         bwd_kv_tile<T, D, NW, true>(p, sm.kv, tile, bh, 0, half);
 }
 
-// Whether the fused launch applies to this dtype and D (both sides one launch shape, one dK / dV part,
-// not fp32 at D = 64); it also needs at most FUSED_MAX slots per head.
+// Whether the fused launch applies to this dtype and D (both sides one launch shape, one dK / dV part);
+// it also needs at most FUSED_MAX slots per head.  fp32 at D = 64 runs one workgroup per CU: as two
+// launches each side lasts at least as long as its heaviest tile, 24 blocks at B2 H12 T1500 where the mean
+// load of a CU is 14.6.  Forward + backward there, two launches -> fused and split: B2 H12 T1500 545 -> 431 us,
+// B1 H4 T4096 1270 -> 552, B4 H12 T2048 1270 -> 1218, B8 H16 T1024 level, B2 H16 T8192 within 1%.
 template <typename T, int D>
 constexpr bool kvq_fused() {
-    return kv_wpe<T, D>() == q_wpe<T, D>() && kv_parts<T, D>() == 1 && !(sizeof(T) == 4 && D == 64);
+    return kv_wpe<T, D>() == q_wpe<T, D>() && kv_parts<T, D>() == 1;
 }
 
 template <typename T, int D>
@@ -90,7 +93,7 @@ static hipError_t launch_kvq_t(const BwdParams &p, hipStream_t s) {
         hipError_t e = launch_bwd_kv(p, sizeof(T) == 2 ? 0 : 1, D, s);
         return e != hipSuccess ? e : launch_bwd_q(p, sizeof(T) == 2 ? 0 : 1, D, s);
     };
-    // No common launch shape, or (fp32 at D = 64, one wave per SIMD) two launches measured 2% faster.
+    // No common launch shape.
     if constexpr (!kvq_fused<T, D>()) {
         return two_launches();
     } else {
