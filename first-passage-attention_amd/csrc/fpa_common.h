@@ -509,6 +509,117 @@ __device__ __forceinline__ void load_row_p1(OpRow<T, D> &dst, const T *rowp, boo
         p1_zero<T, D>(dst);
 }
 
+// ---------------------------------------------------------------------------
+// fp32 products on the bf16 matrix cores.
+//
+// An fp32 value is the sum of three bf16 values, x = h + m + l with h = bf16(x), m = bf16(x - h),
+// l = bf16(x - h - m) rounded to nearest (both differences are exact; what l leaves over is below
+// 2^-26 |x|, and 0 for most x).  A product of two such sums keeps the six terms down to 2^-18 of it
+// (hh, hm, mh, mm, hl, lh); the largest one left out (m l) is below 2^-26, a quarter of an fp32 rounding.
+// The MFMA multiplies bf16 exactly and adds 16 products per step in fp32, so a dot product of D terms takes
+// 6 D / 16 accumulations where the fp32 MFMA (two products per step) takes D / 2.  The 32x32x16 bf16 MFMA
+// has 16 times the fp32 one's rate: 6 of them replace 8 fp32 MFMAs of twice their length each.
+// The five small terms of every step are added first, from zero, and the h h products last, so that only
+// those round at the size of the result; sums over more than one tile are added up outside the MFMA.
+// Infinite operands (and finite ones above 3.39e38) split into NaN: they give NaN where an fp32 product
+// may give an infinity.
+// ---------------------------------------------------------------------------
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+
+struct Split8 {  // eight fp32 values as three bf16 vectors
+    b8 h, m, l;
+};
+__device__ __forceinline__ Split8 split8(f32x8 x) {
+    Split8 r;
+    r.h = __builtin_convertvector(x, b8);
+    x -= __builtin_convertvector(r.h, f32x8);
+    r.m = __builtin_convertvector(x, b8);
+    x -= __builtin_convertvector(r.m, f32x8);
+    r.l = __builtin_convertvector(x, b8);
+    return r;
+}
+
+// A tile of NR rows as three bf16 planes (h, m, l), each with the rows at a pitch of DT + 8 elements
+// (ROWB / 16 odd: conflict-free as Pad's).
+template <int DT, int NR> struct SplitTile {
+    static constexpr int PITCH = DT + 8;
+    static constexpr int PLANE = NR * PITCH * 2;  // bytes
+    static constexpr int BYTES = 3 * PLANE;
+};
+
+// Loads an NR x D fp32 tile into registers (32 contiguous bytes per thread and piece) and, once the tile's
+// last readers have passed a barrier, splits it into LDS planes: each element is split once per
+// workgroup, not once per wave that reads it.
+template <int D, int DT, int NR, int NW> struct SplitLoader {
+    static constexpr int CPR = D / 8, N = NR * CPR, PER = (N + 64 * NW - 1) / (64 * NW);
+    static_assert(N % 64 == 0, "whole waves");
+    f32x4 a[PER], b[PER];
+    // Rows row0 .. row0 + NR - 1 of the tensor whose row 0 is `base`; rows past T_ read row T_ - 1.
+    __device__ __forceinline__ void load(const float *base, int64_t st, int row0, int T_, int tid) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int k = tid + 64 * NW * j, r = min(k, N - 1) / CPR, ch = k % CPR;
+            const float *src = base + (int64_t)min(row0 + r, T_ - 1) * st + 8 * ch;
+            a[j] = *reinterpret_cast<const f32x4 *>(src);
+            b[j] = *reinterpret_cast<const f32x4 *>(src + 4);
+        }
+    }
+    __device__ __forceinline__ void store(char *tile, int tid) const {
+        using S = SplitTile<DT, NR>;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int k = tid + 64 * NW * j, r = k / CPR, ch = k % CPR;
+            if (N % (64 * NW) != 0 && k >= N) break;
+            const Split8 v = split8(__builtin_shufflevector(a[j], b[j], 0, 1, 2, 3, 4, 5, 6, 7));
+            char *dst = tile + (r * S::PITCH + 8 * ch) * 2;
+            *reinterpret_cast<b8 *>(dst) = v.h;
+            *reinterpret_cast<b8 *>(dst + S::PLANE) = v.m;
+            *reinterpret_cast<b8 *>(dst + 2 * S::PLANE) = v.l;
+        }
+    }
+};
+
+__device__ __forceinline__ f32x16 mma_b16(b8 a, b8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+// The accumulator tile c as P2 operands: element e of half hf is register 8 hf + e.
+__device__ __forceinline__ void split_p2(Split8 (&p2)[2], const f32x16 &c) {
+    p2[0] = split8(__builtin_shufflevector(c, c, 0, 1, 2, 3, 4, 5, 6, 7));
+    p2[1] = split8(__builtin_shufflevector(c, c, 8, 9, 10, 11, 12, 13, 14, 15));
+}
+// acc += A B, A the P3 operand of rows row0 .. row0 + 31 of a split tile (column ncol0 + lane % 32), B = p2.
+// The products are summed from zero and added to acc in one rounding.
+template <int DT, int NR>
+__device__ __forceinline__ f32x16 mma_p3_split(f32x16 acc, const Split8 (&p2)[2], const char *tile, int row0, int ncol0,
+                                               int lane) {
+    using S = SplitTile<DT, NR>;
+    const f16 *X = reinterpret_cast<const f16 *>(tile) + row0 * S::PITCH;
+    f32x16 d = zero16();
+    b8 h[2];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+        h[hf] = __builtin_bit_cast(b8, p3_tr(X, S::PITCH, 16 * hf, ncol0, lane));
+        const b8 m = __builtin_bit_cast(b8, p3_tr(X + S::PLANE / 2, S::PITCH, 16 * hf, ncol0, lane));
+        const b8 l = __builtin_bit_cast(b8, p3_tr(X + S::PLANE, S::PITCH, 16 * hf, ncol0, lane));
+        d = mma_b16(l, p2[hf].h, d);
+        d = mma_b16(h[hf], p2[hf].l, d);
+        d = mma_b16(m, p2[hf].m, d);
+        d = mma_b16(m, p2[hf].h, d);
+        d = mma_b16(h[hf], p2[hf].m, d);
+    }
+    d = mma_b16(h[0], p2[0].h, d);
+    d = mma_b16(h[1], p2[1].h, d);
+    return acc + d;
+}
+
+// fp32 operands whose P V runs as split bf16 triples in the forward.  The scores stay on the fp32 MFMA, as the
+// backward recomputes them there and has to round them as the forward did; the backward's products stay there
+// too: split, they were 1.4 times as fast, but the split dP moved dbeta, whose terms cancel, from 1.0e-6 to
+// 1.6e-6 at B2 H12 T1500 D64.
+template <typename T, int D>
+constexpr bool split_fp32() { return sizeof(T) == 4 && D <= 64; }
+
 // Work-item and workgroup ids read from the hardware registers.  (Built with IEEE mode off,
 // the kernels cannot inline the device library's accessors behind threadIdx / blockIdx /
 // gridDim, which then become function calls.)

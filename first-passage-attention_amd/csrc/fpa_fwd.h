@@ -11,6 +11,8 @@
 // row-major tile with LDS transpose reads), and keeps each query's online-softmax state in its own
 // lane.
 #pragma once
+#include <type_traits>
+
 #include "fpa_common.h"
 #include "fpa_params.h"
 
@@ -68,13 +70,16 @@ fpa_fwd_kernel(FwdParams p) {
     constexpr int BM = 32 * NW, BN = 64;
     constexpr int DT = D < 32 ? 32 : D;
     constexpr int NDT = DT / 32;
-    constexpr int TB = Pad<T, DT>::template bytes<BN>();  // one padded K or V tile
+    constexpr bool SP = split_fp32<T, D>();
+    constexpr int TB = SP ? SplitTile<DT, BN>::BYTES : Pad<T, DT>::template bytes<BN>();  // one V tile
     // Two stages when WPE workgroups' worth of them (K, V and the per-key values) fit a CU's 160 KB.
-    constexpr int NS = (WPE * (4 * TB + 2 * 4 * BN * 4) <= 160 * 1024) ? 2 : 1;
-    __shared__ __attribute__((aligned(1024))) char Ks[NS][TB];
+    constexpr int NS = (!SP && WPE * (4 * TB + 2 * 4 * BN * 4) <= 160 * 1024) ? 2 : 1;
+    constexpr int TBK = Pad<T, DT>::template bytes<BN>();  // one K tile
+    constexpr int NC = SP ? 2 : NS;  // stages of the per-key values
+    __shared__ __attribute__((aligned(1024))) char Ks[NS][TBK];
     __shared__ __attribute__((aligned(1024))) char Vs[NS][TB];
     // Per-key values of a tile: CA, CP (SUF, PSI for fp32), PHI and BST (the block's BMIN at [3][0]).
-    __shared__ __attribute__((aligned(1024))) float cst[NS][4][BN];
+    __shared__ __attribute__((aligned(1024))) float cst[NC][4][BN];
 
     const int tid = thread_x(), lane = tid % 64, g = lane / 32, c = lane % 32;
     const int w = __builtin_amdgcn_readfirstlane(tid / 64);  // wave index, uniform across the wave
@@ -115,7 +120,27 @@ fpa_fwd_kernel(FwdParams p) {
     kld.init(p.sk.t, w, lane);
     vld.init(p.sv.t, w, lane);
     const uint32_t aK = lds_addr(&Ks[0][0]), aV = lds_addr(&Vs[0][0]), aC = lds_addr(&cst[0][0][0]);
+    // fp32 at D <= 64: P V on the split path, its V tile through registers (load_split fetches it, store_split
+    // splits it into the planes once its last readers have passed a barrier); K as otherwise.
+    SplitLoader<SP ? D : 32, DT, BN, NW> vsl;
+    auto load_split = [&](int jt, int cbuf) {
+        if constexpr (SP) {
+            buf_lds16(buf_rsrc(st_head + jt * BN), cst_off, aC + cbuf * sizeof(cst[0]));
+            vsl.load(Vb, p.sv.t, jt * BN, p.T, tid);
+        }
+    };
+    auto store_split = [&](int buf) {
+        if constexpr (SP) {
+            vsl.store(Vs[buf], tid);
+        }
+    };
     auto issue = [&](int jt, int buf) {
+        if constexpr (SP) {
+            load_split(jt, buf);
+            kld.issue(aK + buf * sizeof(Ks[0]), Kb, p.sk.t, jt * BN, p.T, w, lane);
+            store_split(buf);
+            return;
+        }
         kld.issue(aK + buf * sizeof(Ks[0]), Kb, p.sk.t, jt * BN, p.T, w, lane);
         vld.issue(aV + buf * sizeof(Vs[0]), Vb, p.sv.t, jt * BN, p.T, w, lane);
         buf_lds16(buf_rsrc(st_head + jt * BN), cst_off, aC + buf * sizeof(cst[0]));
@@ -157,12 +182,15 @@ fpa_fwd_kernel(FwdParams p) {
     wait_loads();
     __syncthreads();
     for (int jt = jhi, it = 0; jt >= jlo; --jt, ++it) {
-        const int buf = (NS == 2) ? (it & 1) : 0;
+        const int buf = (NS == 2) ? (it & 1) : 0, cbuf = (NC == 2) ? (it & 1) : 0;
         const int s0 = jt * BN;
-        if constexpr (NS == 2) issue_full(jt > 0 ? jt - 1 : 0, buf ^ 1);
+        if constexpr (SP)
+            load_split(jt > 0 ? jt - 1 : 0, (it & 1) ^ 1);
+        else if constexpr (NS == 2)
+            issue_full(jt > 0 ? jt - 1 : 0, buf ^ 1);
         if (wave_active && s0 <= qw0 + 31) {
             const char *Kt = Ks[buf];
-            const float *cA = cst[buf][0], *cP = cst[buf][1], *cPHI = cst[buf][2];
+            const float *cA = cst[cbuf][0], *cP = cst[cbuf][1], *cPHI = cst[cbuf][2];
             const int jb = jt;  // BN == G: the key tile is one statistics block
             const bool diag = (jb == ib);
             const float Y = XB ? fminf(pre_t, mid) : betal * fminf(pre_t, mid);
@@ -173,7 +201,7 @@ fpa_fwd_kernel(FwdParams p) {
             f32x16 s[2];
             // Measured: fp16 at D <= 64 (3 waves per SIMD) and fp32 at D = 256 (20 fewer spilled registers,
             // 3% faster); level or slower for the other shapes.
-            constexpr bool SPLIT = FPA_FWD_SPLIT && ((sizeof(T) == 2 && D <= 64) || (sizeof(T) == 4 && D == 256));
+            constexpr bool SPLIT = FPA_FWD_SPLIT && ((sizeof(T) == 2 && D <= 64) || (sizeof(T) == 4 && (D == 256 || SP)));
             if constexpr (!SPLIT) {
                 s[0] = zero16();
                 s[1] = zero16();
@@ -181,7 +209,8 @@ fpa_fwd_kernel(FwdParams p) {
             }
 #pragma unroll
             for (int mt = 1; mt >= 0; --mt) {
-                if constexpr (SPLIT) s[mt] = mma_p1_pad_reg<T, D, DT>(zero16(), Kt, 32 * mt + c, g, qreg);
+                if constexpr (SPLIT)
+                    s[mt] = mma_p1_pad_reg<T, D, DT>(zero16(), Kt, 32 * mt + c, g, qreg);
                 if (!diag) {
 #pragma unroll
                     for (int jq = 0; jq < 4; ++jq) {
@@ -260,18 +289,27 @@ fpa_fwd_kernel(FwdParams p) {
                         rs += pv;
                     }
                     l_i += sum_halves(rs);
+                    Split8 p2[2];
+                    if constexpr (SP) split_p2(p2, s[mt]);
 #pragma unroll
                     for (int dt = 0; dt < NDT; ++dt)
-                        oacc[dt] = mma_p2_p3_pad<T, DT, true>(oacc[dt], s[mt], Vs[buf], 32 * mt, 32 * dt, lane);
+                        if constexpr (SP)
+                            oacc[dt] = mma_p3_split<DT, BN>(oacc[dt], p2, Vs[buf], 32 * mt, 32 * dt, lane);
+                        else
+                            oacc[dt] = mma_p2_p3_pad<T, DT, true>(oacc[dt], s[mt], Vs[buf], 32 * mt, 32 * dt, lane);
                 }
             }
 
-            if (jb < ib) mid = fminf(mid, cst[buf][3][0]);  // BMIN of block jb
+            if (jb < ib) mid = fminf(mid, cst[cbuf][3][0]);  // BMIN of block jb
         }
         if constexpr (NS == 1) {  // every wave is done with the tile: load the next one in its place
             __syncthreads();
-            issue_full(jt > 0 ? jt - 1 : 0, 0);
+            if constexpr (SP)
+                kld.issue_full(aK, Kb, p.sk.t, (jt > 0 ? jt - 1 : 0) * BN, w);
+            else
+                issue_full(jt > 0 ? jt - 1 : 0, 0);
         }
+        if constexpr (SP) store_split(0);
         wait_loads();
         __syncthreads();
     }
