@@ -521,9 +521,12 @@ __device__ __forceinline__ void load_row_p1(OpRow<T, D> &dst, const T *rowp, boo
 // has 16 times the fp32 one's rate: 6 of them replace 8 fp32 MFMAs of twice their length each.
 // The five small terms of every step are added first, from zero, and the h h products last, so that only
 // those round at the size of the result; sums over more than one tile are added up outside the MFMA.
-// Infinite operands (and finite ones above 3.39e38) split into NaN: they give NaN where an fp32 product
-// may give an infinity.
+//
+// Range.  h, m and l have to be finite: a tile that holds a value of 2^64 or more, an infinity among them, stays
+// in fp32 and on the fp32 MFMA (SplitLoader::beyond).
 // ---------------------------------------------------------------------------
+constexpr float SPLIT_MAX = 0x1p64f;
+
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 
@@ -550,7 +553,8 @@ template <int DT, int NR> struct SplitTile {
 
 // Loads an NR x D fp32 tile into registers (32 contiguous bytes per thread and piece) and, once the tile's
 // last readers have passed a barrier, splits it into LDS planes: each element is split once per
-// workgroup, not once per wave that reads it.
+// workgroup, not once per wave that reads it.  store_raw keeps it in fp32, in the layout of Pad<float, DT>,
+// which the planes' space holds.
 template <int D, int DT, int NR, int NW> struct SplitLoader {
     static constexpr int CPR = D / 8, N = NR * CPR, PER = (N + 64 * NW - 1) / (64 * NW);
     static_assert(N % 64 == 0, "whole waves");
@@ -563,6 +567,27 @@ template <int D, int DT, int NR, int NW> struct SplitLoader {
             const float *src = base + (int64_t)min(row0 + r, T_ - 1) * st + 8 * ch;
             a[j] = *reinterpret_cast<const f32x4 *>(src);
             b[j] = *reinterpret_cast<const f32x4 *>(src + 4);
+        }
+    }
+    // Whether any of the wave's elements is too large to split.
+    __device__ __forceinline__ bool beyond() const {
+        float mx = 0.f;
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mx = fmaxf(fmaxf(mx, fabsf(a[j][e])), fabsf(b[j][e]));
+        return __any(mx >= SPLIT_MAX);
+    }
+    __device__ __forceinline__ void store_raw(char *tile, int tid) const {
+        using P = Pad<float, DT>;
+        static_assert(P::template bytes<NR>() <= SplitTile<DT, NR>::BYTES, "the fp32 tile fits the planes");
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int k = tid + 64 * NW * j, r = k / CPR, ch = k % CPR;
+            if (N % (64 * NW) != 0 && k >= N) break;
+            float *dst = reinterpret_cast<float *>(tile) + r * P::PITCH + 8 * ch;
+            *reinterpret_cast<f32x4 *>(dst) = a[j];
+            *reinterpret_cast<f32x4 *>(dst + 4) = b[j];
         }
     }
     __device__ __forceinline__ void store(char *tile, int tid) const {

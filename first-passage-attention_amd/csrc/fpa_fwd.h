@@ -80,6 +80,7 @@ fpa_fwd_kernel(FwdParams p) {
     __shared__ __attribute__((aligned(1024))) char Vs[NS][TB];
     // Per-key values of a tile: CA, CP (SUF, PSI for fp32), PHI and BST (the block's BMIN at [3][0]).
     __shared__ __attribute__((aligned(1024))) float cst[NC][4][BN];
+    __shared__ int vbig[NW];  // split path: whether a wave's part of the V tile in registers is beyond the split's range
 
     const int tid = thread_x(), lane = tid % 64, g = lane / 32, c = lane % 32;
     const int w = __builtin_amdgcn_readfirstlane(tid / 64);  // wave index, uniform across the wave
@@ -120,30 +121,40 @@ fpa_fwd_kernel(FwdParams p) {
     kld.init(p.sk.t, w, lane);
     vld.init(p.sv.t, w, lane);
     const uint32_t aK = lds_addr(&Ks[0][0]), aV = lds_addr(&Vs[0][0]), aC = lds_addr(&cst[0][0][0]);
-    // fp32 at D <= 64: P V on the split path, its V tile through registers (load_split fetches it, store_split
-    // splits it into the planes once its last readers have passed a barrier); K as otherwise.
+    // fp32 at D <= 64: P V on the split path, its V tile through registers (load_split fetches it, vote_split says
+    // whether it can be split, store_split puts it into LDS once its last readers have passed a barrier); K as
+    // otherwise.
     SplitLoader<SP ? D : 32, DT, BN, NW> vsl;
+    bool vraw = false;  // the V tile in LDS is in fp32
     auto load_split = [&](int jt, int cbuf) {
         if constexpr (SP) {
             buf_lds16(buf_rsrc(st_head + jt * BN), cst_off, aC + cbuf * sizeof(cst[0]));
             vsl.load(Vb, p.sv.t, jt * BN, p.T, tid);
         }
     };
-    auto store_split = [&](int buf) {
-        if constexpr (SP) {
-            vsl.store(Vs[buf], tid);
-        }
+    auto vote_split = [&]() { vbig[w] = vsl.beyond(); };
+    auto store_split = [&]() {  // after a barrier that follows the votes
+        int big = 0;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) big |= vbig[i];
+        vraw = __builtin_amdgcn_readfirstlane(big) != 0;
+        if (vraw)
+            vsl.store_raw(Vs[0], tid);
+        else
+            vsl.store(Vs[0], tid);
     };
-    auto issue = [&](int jt, int buf) {
+    auto issue = [&](int jt) {
         if constexpr (SP) {
-            load_split(jt, buf);
-            kld.issue(aK + buf * sizeof(Ks[0]), Kb, p.sk.t, jt * BN, p.T, w, lane);
-            store_split(buf);
-            return;
+            load_split(jt, 0);
+            kld.issue(aK, Kb, p.sk.t, jt * BN, p.T, w, lane);
+            vote_split();
+            __syncthreads();
+            store_split();
+        } else {
+            kld.issue(aK, Kb, p.sk.t, jt * BN, p.T, w, lane);
+            vld.issue(aV, Vb, p.sv.t, jt * BN, p.T, w, lane);
+            buf_lds16(buf_rsrc(st_head + jt * BN), cst_off, aC);
         }
-        kld.issue(aK + buf * sizeof(Ks[0]), Kb, p.sk.t, jt * BN, p.T, w, lane);
-        vld.issue(aV + buf * sizeof(Vs[0]), Vb, p.sv.t, jt * BN, p.T, w, lane);
-        buf_lds16(buf_rsrc(st_head + jt * BN), cst_off, aC + buf * sizeof(cst[0]));
     };
     // Inside the loop every tile loaded is below the first one (jt - 1 < jtmax <= nkt - 1): all rows < T.
     auto issue_full = [&](int jt, int buf) {
@@ -159,7 +170,7 @@ fpa_fwd_kernel(FwdParams p) {
     const int jsplit = (jtmax + 1) >> 1;
     const int jhi = (part == 2) ? jsplit - 1 : jtmax;
     const int jlo = (part == 1) ? jsplit : 0;
-    issue(jhi, 0);
+    issue(jhi);
 
     OpRow<T, D> qreg;
     load_row_p1<T, D>(qreg, Qb + (int64_t)tq * p.sq.t, tq < p.T, g);
@@ -289,27 +300,32 @@ fpa_fwd_kernel(FwdParams p) {
                         rs += pv;
                     }
                     l_i += sum_halves(rs);
-                    Split8 p2[2];
-                    if constexpr (SP) split_p2(p2, s[mt]);
+                    if (SP && !vraw) {
+                        Split8 p2[2];
+                        split_p2(p2, s[mt]);
 #pragma unroll
-                    for (int dt = 0; dt < NDT; ++dt)
-                        if constexpr (SP)
+                        for (int dt = 0; dt < NDT; ++dt)
                             oacc[dt] = mma_p3_split<DT, BN>(oacc[dt], p2, Vs[buf], 32 * mt, 32 * dt, lane);
-                        else
+                    } else {
+#pragma unroll
+                        for (int dt = 0; dt < NDT; ++dt)
                             oacc[dt] = mma_p2_p3_pad<T, DT, true>(oacc[dt], s[mt], Vs[buf], 32 * mt, 32 * dt, lane);
+                    }
                 }
             }
 
             if (jb < ib) mid = fminf(mid, cst[cbuf][3][0]);  // BMIN of block jb
         }
+        if constexpr (SP) vote_split();
         if constexpr (NS == 1) {  // every wave is done with the tile: load the next one in its place
             __syncthreads();
-            if constexpr (SP)
+            if constexpr (SP) {
                 kld.issue_full(aK, Kb, p.sk.t, (jt > 0 ? jt - 1 : 0) * BN, w);
-            else
+                store_split();
+            } else {
                 issue_full(jt > 0 ? jt - 1 : 0, 0);
+            }
         }
-        if constexpr (SP) store_split(0);
         wait_loads();
         __syncthreads();
     }

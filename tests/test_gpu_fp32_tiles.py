@@ -43,3 +43,36 @@ def test_fp32_products_as_bf16_triples(D, scale):
     o = fpa.first_passage_attention(*(t.cuda() for t in (q, k, v, phi, psi, beta)), impl="hip")
     ref = O.fpa_grads(q, k, v, phi, psi, beta, do)[0]
     assert O.rel_err(o.cpu(), ref) <= 2.0 ** -21
+
+
+def _forward(q, k, v, phi, psi, beta):
+    """o from the kernels, and the oracle's in float64."""
+    import fpa
+    o = fpa.first_passage_attention(*(t.cuda() for t in (q, k, v, phi, psi, beta)), impl="hip").cpu()
+    return o, O.fpa_forward(*(t.double() for t in (q, k, v, phi, psi, beta)))
+
+
+@pytest.mark.parametrize("T", [200, 700])  # rows whole, and split in two parts
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("value", [2.0 ** 64, -1e30, 3.4e38, float("inf"), float("-inf")])
+def test_fp32_huge_v(D, T, value):
+    """One value of v at or past the end of what splits into bf16 triples: the rows that see it hold its share
+    (an infinity for an infinity), every other output is as it is without it.  Key 128 starts a tile, so no
+    row before it meets it, not even with weight 0.  The largest finite value takes equal weights, whose sums
+    cannot overflow.  Bounds: 2^-20 for one weight (scores below 2: their rounding and exp2, the row sum, the
+    division, each within 2^-22), 2^-21 in 2-norm as above."""
+    q, k, v, phi, psi, _, _ = O.make_inputs(1, 2, T, D, dtype=torch.float32, seed=73)
+    q = q * (0.0 if value == 3.4e38 else 0.25)
+    beta = torch.zeros(2)
+    base, _ = _forward(q, k, v, phi, psi, beta)
+    v[0, 1, 128, 5] = value
+    o, ref = _forward(q, k, v, phi, psi, beta)
+    seen = o[0, 1, 128:, 5]
+    if abs(value) == float("inf"):
+        assert (seen == value).all()
+    else:
+        want = ref[0, 1, 128:, 5]
+        assert ((seen.double() - want).abs() <= 2.0 ** -20 * want.abs()).all()
+    o[0, 1, 128:, 5] = base[0, 1, 128:, 5]
+    v[0, 1, 128, 5] = 0.0
+    assert torch.isfinite(o).all() and O.rel_err(o, base) <= 2.0 ** -21
