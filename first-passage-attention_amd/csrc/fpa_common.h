@@ -400,16 +400,18 @@ template <typename T, int D, int DT, int NR, int NW> struct TileLoader {
         const int pc = k % P::CPRP;
         lc = (pc < CPRD) ? pc : pc % CPRD;
     }
-    __device__ __forceinline__ void init(int64_t st, int wave, int lane) {
+    // T_: the tensor's rows, for a loop that calls issue_full also for a first tile of fewer than NR rows.
+    __device__ __forceinline__ void init(int64_t st, int wave, int lane, int T_ = NR) {
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             int r, lc;
             slot(min(wave + NW * j, NI - 1), lane, r, lc);
-            off[j] = (uint32_t)((r * st + lc * P::CE) * (int64_t)sizeof(T));
+            off[j] = (uint32_t)((min(r, T_ - 1) * st + lc * P::CE) * (int64_t)sizeof(T));
         }
     }
-    // issue() for a tile whose rows are all below T: no per-lane clamping, so a loop that only loads
-    // such tiles keeps no clamped offsets live.
+    // issue() for a tile whose rows are all below T (or, with T_ given to init, the first tile: rows past
+    // T read row T - 1): no per-lane clamping, so a loop that only loads such tiles keeps no clamped offsets
+    // live.
     __device__ __forceinline__ void issue_full(uint32_t tile, const T *base, int64_t st, int row0, int wave) const {
         const u32x4 rs = buf_rsrc(base + (int64_t)row0 * st);
 #pragma unroll

@@ -118,8 +118,8 @@ fpa_fwd_kernel(FwdParams p) {
     // issues the per-key load, identical writes instead of a wave-dependent branch).  After tile 0
     // the prefetch repeats it into a buffer that is not read again.
     TileLoader<T, D, DT, BN, NW> kld, vld;
-    kld.init(p.sk.t, w, lane);
-    vld.init(p.sv.t, w, lane);
+    kld.init(p.sk.t, w, lane, p.T);
+    vld.init(p.sv.t, w, lane, p.T);
     const uint32_t aK = lds_addr(&Ks[0][0]), aV = lds_addr(&Vs[0][0]), aC = lds_addr(&cst[0][0][0]);
     // fp32 at D <= 64: P V on the split path, its V tile through registers (load_split fetches it, vote_split says
     // whether it can be split, store_split puts it into LDS once its last readers have passed a barrier); K as
@@ -156,7 +156,8 @@ fpa_fwd_kernel(FwdParams p) {
             buf_lds16(buf_rsrc(st_head + jt * BN), cst_off, aC);
         }
     };
-    // Inside the loop every tile loaded is below the first one (jt - 1 < jtmax <= nkt - 1): all rows < T.
+    // Inside the loop every tile loaded is below the first one (jt - 1 < jtmax <= nkt - 1): all rows < T.  Tile 0,
+    // which the last prefetch repeats, may be the first one: at T < 64 the loaders' offsets end at row T - 1.
     auto issue_full = [&](int jt, int buf) {
         kld.issue_full(aK + buf * sizeof(Ks[0]), Kb, p.sk.t, jt * BN, w);
         vld.issue_full(aV + buf * sizeof(Vs[0]), Vb, p.sv.t, jt * BN, w);

@@ -126,3 +126,21 @@ def test_split_only_where_the_launch_is_short():
     assert split_tiles(16, 4096, 1, 128) == 0       # cfg3: 512 workgroups, 512 slots
     assert split_tiles(12, 16381, 0, 64) == 0       # cfg4
     assert split_tiles(2, 384, 0, 64) == 0          # three row tiles
+
+
+@pytest.mark.parametrize("T", [1, 17, 63, 64, 65, 127, 128, 129, 513, 1000])
+def test_every_row_loaded_is_below_T(T):
+    """The rows of K and V that an item loads: its first tile clamped to T - 1 (TileLoader::issue), the prefetched ones
+    by offsets fixed before the loop (issue_full), where the last prefetch repeats tile 0."""
+    nqt, nkt = (T + BM - 1) // BM, (T + BN - 1) // BN
+    offsets = [min(r, T - 1) for r in range(BN)]  # TileLoader::init with the tensor's rows
+    for ns in {0, split_tiles(1, T, 0, 64)}:
+        for k in range(nqt + ns):
+            rank, part = decode(k, ns)
+            jtmax = min(nkt - 1, ((nqt - 1 - rank) * BM + BM - 1) // BN)
+            jsplit = (jtmax + 1) >> 1
+            jhi, jlo = (jsplit - 1 if part == 2 else jtmax), (jsplit if part == 1 else 0)
+            assert jhi * BN < T
+            for jt in range(jhi, jlo - 1, -1):
+                nxt = jt - 1 if jt > 0 else 0
+                assert max(nxt * BN + r for r in offsets) < T
