@@ -512,7 +512,8 @@ __device__ __forceinline__ void load_row_p1(OpRow<T, D> &dst, const T *rowp, boo
 }
 
 // ---------------------------------------------------------------------------
-// fp32 products on the bf16 matrix cores.
+// fp32 products on the bf16 matrix cores (the three-term bfloat16 split of Henry, Tang and Heinecke,
+// "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", 2019).
 //
 // An fp32 value is the sum of three bf16 values, x = h + m + l with h = bf16(x), m = bf16(x - h),
 // l = bf16(x - h - m) rounded to nearest (both differences are exact; what l leaves over is below
@@ -524,19 +525,23 @@ __device__ __forceinline__ void load_row_p1(OpRow<T, D> &dst, const T *rowp, boo
 // The five small terms of every step are added first, from zero, and the h h products last, so that only
 // those round at the size of the result; sums over more than one tile are added up outside the MFMA.
 //
-// Range.  h, m and l have to be finite: a tile that holds a value of 2^64 or more, an infinity among them, stays
-// in fp32 and on the fp32 MFMA (SplitLoader::beyond).
+// Range.  h, m and l have to be finite and normal.  Both operands are scaled by 2^24, so that the lowest bit
+// of any fp32 value, 2^-149, becomes 2^-125: the split of every x below SPLIT_MAX = 2^64 is as exact as that
+// of 1 (the scaling itself is exact, and taken out as the products are added to the result).  P is at most
+// 2^RESCALE_SLACK = 2^8, so that 32 products stay below 2^(24 + 64 + 24 + 8 + 5) = 2^125.  A tile that holds a larger
+// value, an infinity among them, stays in fp32 and on the fp32 MFMA (SplitLoader::beyond).
 // ---------------------------------------------------------------------------
-constexpr float SPLIT_MAX = 0x1p64f;
+constexpr float SPLIT_SCALE = 0x1p24f, SPLIT_UNSCALE = 0x1p-48f, SPLIT_MAX = 0x1p64f;
 
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 
-struct Split8 {  // eight fp32 values as three bf16 vectors
+struct Split8 {  // eight fp32 values, times SPLIT_SCALE, as three bf16 vectors
     b8 h, m, l;
 };
 __device__ __forceinline__ Split8 split8(f32x8 x) {
     Split8 r;
+    x *= SPLIT_SCALE;
     r.h = __builtin_convertvector(x, b8);
     x -= __builtin_convertvector(r.h, f32x8);
     r.m = __builtin_convertvector(x, b8);
@@ -616,7 +621,7 @@ __device__ __forceinline__ void split_p2(Split8 (&p2)[2], const f32x16 &c) {
     p2[1] = split8(__builtin_shufflevector(c, c, 8, 9, 10, 11, 12, 13, 14, 15));
 }
 // acc += A B, A the P3 operand of rows row0 .. row0 + 31 of a split tile (column ncol0 + lane % 32), B = p2.
-// The products are summed from zero and added to acc in one rounding.
+// The products are summed from zero and added to acc, the operands' scaling taken out, in one rounding.
 template <int DT, int NR>
 __device__ __forceinline__ f32x16 mma_p3_split(f32x16 acc, const Split8 (&p2)[2], const char *tile, int row0, int ncol0,
                                                int lane) {
@@ -637,7 +642,9 @@ __device__ __forceinline__ f32x16 mma_p3_split(f32x16 acc, const Split8 (&p2)[2]
     }
     d = mma_b16(h[0], p2[0].h, d);
     d = mma_b16(h[1], p2[1].h, d);
-    return acc + d;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[j] = fmaf(d[j], SPLIT_UNSCALE, acc[j]);
+    return acc;
 }
 
 // fp32 operands whose P V runs as split bf16 triples in the forward.  The scores stay on the fp32 MFMA, as the

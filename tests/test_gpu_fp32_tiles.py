@@ -60,7 +60,7 @@ def test_fp32_huge_v(D, T, value):
     (an infinity for an infinity), every other output is as it is without it.  Key 128 starts a tile, so no
     row before it meets it, not even with weight 0.  The largest finite value takes equal weights, whose sums
     cannot overflow.  Bounds: 2^-20 for one weight (scores below 2: their rounding and exp2, the row sum, the
-    division, each within 2^-22), 2^-21 in 2-norm as above."""
+    division, each within 2^-22), 2^-21 of the largest output as above."""
     q, k, v, phi, psi, _, _ = O.make_inputs(1, 2, T, D, dtype=torch.float32, seed=73)
     q = q * (0.0 if value == 3.4e38 else 0.25)
     beta = torch.zeros(2)
@@ -76,3 +76,27 @@ def test_fp32_huge_v(D, T, value):
     o[0, 1, 128:, 5] = base[0, 1, 128:, 5]
     v[0, 1, 128, 5] = 0.0
     assert torch.isfinite(o).all() and O.rel_err(o, base) <= 2.0 ** -21
+
+
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("scale", [1e-30, 1e-33, 1e-36])
+def test_fp32_tiny_v(D, scale):
+    """Values whose bf16 triples would be subnormal: o (down to 1e-37, still normal) is within the same 2^-21."""
+    q, k, v, phi, psi, beta, _ = O.make_inputs(1, 2, 500, D, dtype=torch.float32, seed=74)
+    o, ref = _forward(q, k, v * scale, phi, psi, beta)
+    assert O.rel_err(o.double() / scale, ref / scale) <= 2.0 ** -21
+
+
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("value", [1.0, 2.0 ** 60, 2.0 ** 100])
+def test_fp32_tiny_weight(D, value):
+    """A weight of 2^-124 (score -86) on the only nonzero value: its share is o.  Bound 2^-15: the score, 124 in base 2,
+    and its scaling round by 2^-17 each, which exp2 turns into a relative error."""
+    q = torch.zeros(1, 1, 3, D)
+    k, v = torch.zeros_like(q), torch.zeros_like(q)
+    q[..., 0] = 8.0
+    k[0, 0, 0, 0] = -86.0 * D ** 0.5 / 8.0
+    v[0, 0, 0, 3] = value
+    zero = torch.zeros(1, 1, 3)
+    o, ref = _forward(q, k, v, zero, zero, torch.zeros(1))
+    assert ((o.double() - ref)[0, 0, 2].abs() <= 2.0 ** -15 * ref[0, 0, 2].abs()).all()
