@@ -539,15 +539,30 @@ typedef float f32x8 __attribute__((ext_vector_type(8)));
 struct Split8 {  // eight fp32 values, times SPLIT_SCALE, as three bf16 vectors
     b8 h, m, l;
 };
-__device__ __forceinline__ Split8 split8(f32x8 x) {
-    Split8 r;
-    x *= SPLIT_SCALE;
-    r.h = __builtin_convertvector(x, b8);
-    x -= __builtin_convertvector(r.h, f32x8);
-    r.m = __builtin_convertvector(x, b8);
-    x -= __builtin_convertvector(r.m, f32x8);
-    r.l = __builtin_convertvector(x, b8);
+// A pair rounded by one conversion, to be widened again by a shift and a mask.  The empty asm hides where the bits
+// come from: the compiler otherwise rounds every element a second time, alone, to widen it (32 conversions more for
+// 16 values).
+__device__ __forceinline__ uint32_t round_pair(float a, float b) {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    uint32_t r = __builtin_bit_cast(uint32_t, b2{(__bf16)a, (__bf16)b});
+    asm("" : "+v"(r));
     return r;
+}
+__device__ __forceinline__ Split8 split8(f32x8 x) {
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    u32x4_t h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = x[2 * i] * SPLIT_SCALE, b = x[2 * i + 1] * SPLIT_SCALE;
+        h[i] = round_pair(a, b);
+        a -= __uint_as_float(h[i] << 16);
+        b -= __uint_as_float(h[i] & 0xffff0000u);
+        m[i] = round_pair(a, b);
+        a -= __uint_as_float(m[i] << 16);
+        b -= __uint_as_float(m[i] & 0xffff0000u);
+        l[i] = round_pair(a, b);
+    }
+    return Split8{__builtin_bit_cast(b8, h), __builtin_bit_cast(b8, m), __builtin_bit_cast(b8, l)};
 }
 
 // A tile of NR rows as three bf16 planes (h, m, l), each with the rows at a pitch of DT + 8 elements
@@ -566,14 +581,15 @@ template <int D, int DT, int NR, int NW> struct SplitLoader {
     static constexpr int CPR = D / 8, N = NR * CPR, PER = (N + 64 * NW - 1) / (64 * NW);
     static_assert(N % 64 == 0, "whole waves");
     f32x4 a[PER], b[PER];
-    // Rows row0 .. row0 + NR - 1 of the tensor whose row 0 is `base`; rows past T_ read row T_ - 1.
-    __device__ __forceinline__ void load(const float *base, int64_t st, int row0, int T_, int tid) {
+    // The tile whose first row is at `src` (wave-uniform); its rows from `rows` on read row rows - 1.  The offsets
+    // from src fit 32 bits, as TileLoader's do, and stay in registers where `rows` is the same for every tile.
+    __device__ __forceinline__ void load(const float *src, int64_t st, int rows, int tid) {
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             const int k = tid + 64 * NW * j, r = min(k, N - 1) / CPR, ch = k % CPR;
-            const float *src = base + (int64_t)min(row0 + r, T_ - 1) * st + 8 * ch;
-            a[j] = *reinterpret_cast<const f32x4 *>(src);
-            b[j] = *reinterpret_cast<const f32x4 *>(src + 4);
+            const uint32_t off = (uint32_t)((min(r, rows - 1) * st + 8 * ch) * 4);
+            a[j] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(src) + off);
+            b[j] = *reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(src) + off + 16);
         }
     }
     // Whether any of the wave's elements is too large to split.
@@ -647,10 +663,14 @@ __device__ __forceinline__ f32x16 mma_p3_split(f32x16 acc, const Split8 (&p2)[2]
     return acc;
 }
 
-// fp32 operands whose P V runs as split bf16 triples in the forward.  The scores stay on the fp32 MFMA, as the
-// backward recomputes them there and has to round them as the forward did; the backward's products stay there
-// too: split, they were 1.4 times as fast, but the split dP moved dbeta, whose terms cancel, from 1.0e-6 to
-// 1.6e-6 at B2 H12 T1500 D64.
+// fp32 operands whose P V runs as split bf16 triples in the forward: D <= 64.  Forward on the fp32 MFMA -> split at
+// B4 H12 T2048: D = 64 256 -> 216 us, 32 142 -> 131, 16 117 -> 108; at B1 H2 T3000, one wave per SIMD, where the
+// splitting of P costs as much as its products save, 32 82 -> 84 and 16 71 -> 71.  o is off by half as much
+// (2-norm against float64, T 256 to 4096: 2.4e-7 .. 4.6e-7 -> 1.5e-7 .. 2.5e-7).  At D = 128 the V planes (52 KB) and
+// K (34 KB) of two workgroups pass the 160 KB of a CU.
+// The scores stay on the fp32 MFMA, as the backward recomputes them there and has to round them as the
+// forward did; the backward's products stay there too: split, they were 1.4 times as fast, but the split dP moved
+// dbeta, whose terms cancel, from 1.0e-6 to 1.6e-6 at B2 H12 T1500 D64.
 template <typename T, int D>
 constexpr bool split_fp32() { return sizeof(T) == 4 && D <= 64; }
 

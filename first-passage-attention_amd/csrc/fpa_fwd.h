@@ -126,10 +126,10 @@ fpa_fwd_kernel(FwdParams p) {
     // otherwise.
     SplitLoader<SP ? D : 32, DT, BN, NW> vsl;
     bool vraw = false;  // the V tile in LDS is in fp32
-    auto load_split = [&](int jt, int cbuf) {
+    auto load_split = [&](int jt, int rows, int cbuf) {
         if constexpr (SP) {
             buf_lds16(buf_rsrc(st_head + jt * BN), cst_off, aC + cbuf * sizeof(cst[0]));
-            vsl.load(Vb, p.sv.t, jt * BN, p.T, tid);
+            vsl.load(Vb + (int64_t)jt * BN * p.sv.t, p.sv.t, rows, tid);
         }
     };
     auto vote_split = [&]() { vbig[w] = vsl.beyond(); };
@@ -145,7 +145,7 @@ fpa_fwd_kernel(FwdParams p) {
     };
     auto issue = [&](int jt) {
         if constexpr (SP) {
-            load_split(jt, 0);
+            load_split(jt, p.T - jt * BN, 0);
             kld.issue(aK, Kb, p.sk.t, jt * BN, p.T, w, lane);
             vote_split();
             __syncthreads();
@@ -197,7 +197,7 @@ fpa_fwd_kernel(FwdParams p) {
         const int buf = (NS == 2) ? (it & 1) : 0, cbuf = (NC == 2) ? (it & 1) : 0;
         const int s0 = jt * BN;
         if constexpr (SP)
-            load_split(jt > 0 ? jt - 1 : 0, (it & 1) ^ 1);
+            load_split(jt > 0 ? jt - 1 : 0, p.T, (it & 1) ^ 1);
         else if constexpr (NS == 2)
             issue_full(jt > 0 ? jt - 1 : 0, buf ^ 1);
         if (wave_active && s0 <= qw0 + 31) {
