@@ -77,12 +77,22 @@ fpa_bwd_kvq_split_kernel(BwdParams p, BwdOrder ord, int nslots) {
 
 // Whether the fused launch applies to this dtype and D (both sides one launch shape, one dK / dV part);
 // it also needs at most FUSED_MAX slots per head.  fp32 at D = 64 runs one workgroup per CU: as two
-// launches each side lasts at least as long as its heaviest tile, 24 blocks at B2 H12 T1500 where the mean
-// load of a CU is 14.6.  Forward + backward there, two launches -> fused and split: B2 H12 T1500 545 -> 431 us,
-// B1 H4 T4096 1270 -> 552, B4 H12 T2048 1270 -> 1218, B8 H16 T1024 level, B2 H16 T8192 within 1%.
+// launches each side lasts at least as long as its heaviest tile, 24 blocks at 24 heads of T = 1500 where the mean
+// load of a CU is 14.6.  Backward alone there, two launches -> fused: 24 heads of T = 1500 436 -> 307 us, of 2048
+// 575 -> 511, 33 heads of 512 167 -> 101, 12 heads of 8192 3661 -> 3442; -> fused and split: 16 heads of 1024
+// 301 -> 130, 4 heads of 4096 1096 -> 378, 2 heads of 385 (the shortest length that is split) 139 -> 106.
 template <typename T, int D>
 constexpr bool kvq_fused() {
     return kv_wpe<T, D>() == q_wpe<T, D>() && kv_parts<T, D>() == 1;
+}
+
+// One workgroup per CU and an even number of full rounds on each side: heaviest first, every CU gets heavy and light
+// tiles that add up to the same load, and two launches have nothing to gain from each other.  fp32 at D = 64, fused
+// -> two launches: 32 heads of T = 2048 (two rounds a side) 661 -> 636 us, 16 of 4096 1229 -> 1204, 64 of 2048 (four)
+// 1260 -> 1247, 32 of 4096 2358 -> 2326, 64 of 1024 level; at three rounds two launches are 5-6% slower.
+template <typename T, int D>
+constexpr bool pairs_evenly(int64_t tiles) {
+    return sizeof(T) == 4 && D == 64 && tiles % (2 * 8 * XCD_CUS) == 0;
 }
 
 template <typename T, int D>
@@ -97,7 +107,7 @@ static hipError_t launch_kvq_t(const BwdParams &p, hipStream_t s) {
     if constexpr (!kvq_fused<T, D>()) {
         return two_launches();
     } else {
-        if (2 * nt > FUSED_MAX) return two_launches();
+        if (2 * nt > FUSED_MAX || pairs_evenly<T, D>((int64_t)p.BH * nt)) return two_launches();
         // Block iterations of key tile kt (query blocks from its diagonal block to the end) and of
         // query tile qt (key blocks from its diagonal block down to 0), weighted by their cost.
         auto c_kv = [&](int kt) { return FPA_FUSE_WKV * (p.NB - kt * BT / G); };

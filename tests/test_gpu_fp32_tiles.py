@@ -14,6 +14,7 @@ NAMES = ("o", "dq", "dk", "dv", "dphi", "dpsi", "dbeta")
     (1, 2, 449, 64),     # four tiles per side: the first length whose backward is split, one row in the last block
     (2, 4, 1000, 64),    # split, heads pinned to XCDs
     (1, 33, 512, 64),    # four tiles, 264 items: more than the one round that splits
+    (1, 128, 512, 64),   # 512 tiles a side, two rounds: two launches
     (1, 1, 1, 64),       # one row: every other row of its tiles is a copy of it
     (1, 2, 129, 32),     # a second workgroup of one row
     (1, 2, 300, 16),     # half-width operands: columns 16 .. 31 of the tiles are never written
