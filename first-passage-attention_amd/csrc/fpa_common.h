@@ -549,8 +549,7 @@ __device__ __forceinline__ uint32_t round_pair(float a, float b) {
     return r;
 }
 __device__ __forceinline__ Split8 split8(f32x8 x) {
-    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-    u32x4_t h, m, l;
+    u32x4 h, m, l;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         float a = x[2 * i] * SPLIT_SCALE, b = x[2 * i + 1] * SPLIT_SCALE;

@@ -11,8 +11,6 @@
 // row-major tile with LDS transpose reads), and keeps each query's online-softmax state in its own
 // lane.
 #pragma once
-#include <type_traits>
-
 #include "fpa_common.h"
 #include "fpa_params.h"
 

@@ -26,7 +26,7 @@ def kv_wpe(dtype, D):
 
 
 def fused(dtype, D):
-    return D < 256 and not (dtype == 1 and D == 64)   # kv_wpe == q_wpe, one dK/dV part, not fp32 D64
+    return D < 256                                    # kv_wpe == q_wpe, one dK/dV part
 
 
 def split_tiles(BH, T, dtype, D):
@@ -49,7 +49,8 @@ def q_range(qt, NB, half):
 
 
 SHAPES = [(1, 3, 1000, 0, 32), (2, 4, 600, 0, 64), (3, 5, 777, 1, 16), (1, 1, 513, 0, 16), (1, 1, 4100, 0, 128),
-          (1, 2, 777, 1, 32), (1, 4, 4096, 0, 64), (1, 1, 16384, 0, 64), (4, 12, 2048, 0, 64), (1, 2, 385, 0, 64)]
+          (1, 2, 777, 1, 32), (1, 4, 4096, 0, 64), (1, 1, 16384, 0, 64), (4, 12, 2048, 0, 64), (1, 2, 385, 0, 64),
+          (1, 2, 385, 1, 64), (2, 4, 1000, 1, 64), (1, 4, 4096, 1, 64), (2, 12, 1500, 1, 64)]
 
 
 @pytest.mark.parametrize("B,H,T,dtype,D", SHAPES)
@@ -111,5 +112,7 @@ def test_split_only_where_the_launch_is_short():
     assert split_tiles(8, 2048, 0, 64) == (8, 8)     # B1 H8: 256 items
     assert split_tiles(4, 4096, 0, 64) == (16, 16)
     assert split_tiles(48, 2048, 0, 64) == (0, 0)    # cfg2
-    assert split_tiles(2, 1300, 1, 64) == (0, 0)     # fp32 D64 runs the two sides as two launches
+    assert split_tiles(2, 1300, 1, 64) == (5, 5)     # fp32 D64: 44 items of 256 slots
+    assert split_tiles(4, 4096, 1, 64) == (16, 16)   # all 256
+    assert split_tiles(24, 1500, 1, 64) == (0, 0)    # 576 items
     assert split_tiles(1, 384, 0, 64) == (0, 0)      # three tiles

@@ -11,7 +11,8 @@ NAMES = ("o", "dq", "dk", "dv", "dphi", "dpsi", "dbeta")
 
 @pytest.mark.parametrize("B,H,T,D", [
     (1, 1, 65, 64),      # one tile per side, one key past a block
-    (1, 2, 449, 64),     # four tiles per side: the first length whose backward is split, one row in the last block
+    (1, 2, 385, 64),     # four tiles per side, the last of one row: the first length whose backward is split
+    (1, 2, 449, 64),     # four tiles per side, one row in the last block
     (2, 4, 1000, 64),    # split, heads pinned to XCDs
     (1, 33, 512, 64),    # four tiles, 264 items: more than the one round that splits
     (1, 128, 512, 64),   # 512 tiles a side, two rounds: two launches
@@ -20,7 +21,8 @@ NAMES = ("o", "dq", "dk", "dv", "dphi", "dpsi", "dbeta")
     (1, 2, 300, 16),     # half-width operands: columns 16 .. 31 of the tiles are never written
 ])
 def test_fp32_gradients(B, H, T, D):
-    """All outputs within 2e-4 (2-norm), the bound the repository holds its fp32 path to; they are at 3e-6."""
+    """Largest difference over the largest value: within 1e-5, five times the largest of these shapes (1.9e-6); dbeta, whose
+    terms cancel, within 2e-4, the bound the repository holds its fp32 path to."""
     import fpa
     a = O.make_inputs(B, H, T, D, dtype=torch.float32, seed=71, psi_noise=1.0)
     leaves = [t.cuda().requires_grad_() for t in a[:6]]
@@ -30,14 +32,14 @@ def test_fp32_gradients(B, H, T, D):
     for name, x, r in zip(NAMES, got, ref):
         # an exactly zero gradient (dq, dk, dphi, ... of a single row) is checked absolutely: the operands are of order 1
         err = O.rel_err(x.cpu(), r) if r.abs().max() > 0 else x.abs().max().item()
-        assert err <= 2e-4, name
+        assert err <= (2e-4 if name == "dbeta" else 1e-5), name
 
 
 @pytest.mark.parametrize("D", [16, 32, 64])
 @pytest.mark.parametrize("scale", [1e-12, 1.0, 1e4])
 def test_fp32_products_as_bf16_triples(D, scale):
-    """The fp32 products run on the bf16 matrix cores as sums of three-term splits, in each of which 2^-26 of a
-    product is left out: o is within 2^-21 of the oracle, sixteen roundings of an fp32 result, at any size of v."""
+    """P V runs on the bf16 matrix cores as sums of three-term splits, in which 2^-26 of a product is left out: o is
+    within 2^-21 of the oracle, eight roundings of an fp32 result, as it is without them."""
     import fpa
     q, k, v, phi, psi, beta, do = O.make_inputs(1, 2, 500, D, dtype=torch.float32, seed=72, psi_noise=1.0)
     v = v * scale
