@@ -8,7 +8,8 @@
 //   softmax uses exp2 and the saved row statistic lse2 is a base-2 log-sum-exp.
 // * Matrix products run on the 32x32 MFMA of gfx950:
 //     fp16: v_mfma_f32_32x32x16_f16  (one K step contracts 16 indices)
-//     fp32: v_mfma_f32_32x32x2_f32   (one K step contracts 2 indices)
+//     fp32: v_mfma_f32_32x32x2_f32   (one K step contracts 2 indices); the forward's P V at D <= 64
+//           as split bf16 triples on v_mfma_f32_32x32x16_bf16 (split_fp32 below)
 //   Lane l = 32 * g + c (g = l / 32, c = l % 32).  A operand: lane holds row c;
 //   B operand: lane holds column c; lane group g holds its half of the K step.
 //   The 32x32 accumulator: register j of lane l is C[8*(j/4) + 4*g + j%4][c].

@@ -4,19 +4,21 @@
 //
 // Reference behaviour: kernel.py:103-162 (_fwd) of yliu-fort/first-passage-attention.
 // gfx950 design: a workgroup of FPA_NW waves owns 32 query rows per wave, streams 64-key tiles
-// from the diagonal down to key 0 through double-buffered (single-buffered for fp32 at D = 128 and 256,
-// where two stages of the workgroups that share a CU do not fit in LDS), padded LDS tiles filled by
-// direct global->LDS loads (one
-// barrier per tile), computes S^T = K Q^T and O^T += V^T P^T on the 32x32 MFMA (V^T read from the
-// row-major tile with LDS transpose reads), and keeps each query's online-softmax state in its own
-// lane.
+// from the diagonal down to key 0 through padded LDS tiles filled by direct global->LDS loads (fp16:
+// double-buffered, one barrier per tile; fp32: single-buffered, two barriers), computes S^T = K Q^T and
+// O^T += V^T P^T on the 32x32 MFMA (V^T read from the row-major tile with LDS transpose reads), and keeps
+// each query's online-softmax state in its own lane.
+// fp32 at D = 128 and 256 is single-buffered because two stages of the workgroups that share a CU do not
+// fit in LDS; at D <= 64 V passes through registers into split planes, of which there is one stage.  K in two
+// stages there (64.5 KB at D = 64) was measured and changed nothing: B4 H12 T2048 D64 221 -> 225 us, D32 137 -> 139,
+// B1 H2 T3000 D32 88 -> 89; nor did two stages of both at D <= 32 (D32 137 -> 140, B1 H2 T3000 88 -> 92).
 #pragma once
 #include "fpa_common.h"
 #include "fpa_params.h"
 
 // Tuning knobs (build-time): waves per SIMD of the D <= 64 forward kernel, fp16 and fp32 (fp32 at D <= 32
 // runs three: fwd_wpe).  Three fp16 waves fit in 168 VGPRs each; with 3 workgroups per CU the cfg2 grid
-// (768 workgroups) is resident at once.  The fp32 D = 64 kernel needs about 180 VGPRs.
+// (768 workgroups) is resident at once.  The fp32 D = 64 kernel needs 240 VGPRs.
 #ifndef FPA_FWD_WPE
 #define FPA_FWD_WPE 3
 #endif
@@ -24,8 +26,8 @@
 #define FPA_FWD_WPE32 2
 #endif
 // The scores of each 32-key half computed just before its softmax instead of both halves' MFMA chains
-// interleaved up front: fp16 at D <= 64 (13 fewer live registers at D = 64, 1-4% faster at cfg2) and
-// fp32 at D = 256 (see the kernel).
+// interleaved up front: fp16 at D <= 64 (13 fewer live registers at D = 64, 1-4% faster at cfg2), fp32 at
+// D = 256 and fp32 at D <= 64 (see the kernel).
 #ifndef FPA_FWD_SPLIT
 #define FPA_FWD_SPLIT 1
 #endif
@@ -210,7 +212,9 @@ fpa_fwd_kernel(FwdParams p) {
             // and the first half's P V run while the other half's VALU work goes on).
             f32x16 s[2];
             // Measured: fp16 at D <= 64 (3 waves per SIMD) and fp32 at D = 256 (20 fewer spilled registers,
-            // 3% faster); level or slower for the other shapes.
+            // 3% faster); level or slower for the other shapes.  On the split path level at D = 64 (216 us
+            // against 215 at B4 H12 T2048) and 32, and without the one spill at D = 16 and 32 (B1 H2 T3000 D16
+            // 71.3 against 72.8).
             constexpr bool SPLIT = FPA_FWD_SPLIT && ((sizeof(T) == 2 && D <= 64) || (sizeof(T) == 4 && (D == 256 || SP)));
             if constexpr (!SPLIT) {
                 s[0] = zero16();
@@ -417,8 +421,9 @@ __global__ void __launch_bounds__(256) fpa_fwd_merge_kernel(FwdParams p) {
 // stages of K and V (70 KB per workgroup), fp32 in 256 with one register spilled outside the tile loop
 // and one stage (67 KB).  Against one wave per SIMD, whose 512-register budget the compiler had filled
 // (332 and 352 VGPRs): fp16 121 -> 85 us and fp32 531 -> 461 us at B4 H12 T2048, fp32 629 -> 593 us
-// at B2 H8 T4096.  fp32 at D <= 32 fits three (141 and 152 VGPRs, no spills): 6-7% faster than two at
-// B4 H12 T2048 and B2 H8 T4096.
+// at B2 H8 T4096.  fp32 at D <= 32 fits three (166 and 164 VGPRs, no spills): 4-6% faster than two at
+// B4 H12 T2048 and B2 H8 T8192 (D16 112 -> 107 us, D32 138 -> 131), 1-2% slower at B1 H2 T3000, where each SIMD
+// has one wave.
 template <typename T, int D>
 constexpr int fwd_wpe() {
     return (D == 128) ? 2 : (D >= 128) ? 1 : (sizeof(T) == 2 ? FPA_FWD_WPE : (D <= 32 ? 3 : FPA_FWD_WPE32));
